@@ -33,22 +33,61 @@ inline int packedCoBlocks(int cout) { return ceilDiv(ceilDiv(cout, kCoBlock), 8)
 std::vector<float> packConv3x3(const float* w, int cin, int cout);
 size_t packedConv3x3Floats(int cin, int cout);
 
-// A tower convolution's weights w [cout][cin][3][3] (device memory) split in
-// two f16 parts (azh_tower.hpp) on the GPU: w * 2^wexp[co] = h + l, the
-// power of two taking the channel's largest weight into [2^14, 2^15). out:
-// the parts packed as the MFMA A fragments the kernel loads, [co block]
-// [chunk q][tap t][part h, l][lane 0..63][j 0..7], value w[cb*16 + (lane &
-// 15)][q*32 + 8*(lane >> 4) + j][t], zero where the channel is padding (co
-// blocks = packedCoBlocks(cout), chunks = ceil(cin/32));
-// packedTowerFloats(cin, cout) floats' worth. wexp: cout powers of two,
-// kNoSplit added for a channel with an infinity or a NaN (its parts then
-// hold them, and a zero), and at [cout] whether there is such a channel.
-// `layers` such convolutions at once: w one after the other, out and wexp
-// `stride` words apart.
+// A tower layer's weights on the device.
+// parts: the weights w [cout][cin][3][3] split in two f16 parts
+// (azh_tower.hpp), w * 2^wexp[co] = h + l, the power of two taking the
+// channel's largest finite weight into [2^14, 2^15), packed as the MFMA A
+// fragments the kernel loads: [co block][chunk q][tap t][part h, l][lane
+// 0..63][j 0..7], value w[cb*16 + (lane & 15)][q*32 + 8*(lane >> 4) + j][t],
+// zero where the channel is padding (co blocks = packedCoBlocks(cout), chunks
+// = ceil(cin/32)) or the weight an infinity or a NaN.
+// wexp: cout powers of two, kNoSplit added for a channel with an infinity or
+// a NaN among its weights.
+// rest: of the weights that the parts miss by more than 2^-23 of them (2^-16
+// and less of the channel's largest), the difference: kRests a channel, in
+// the order of their index c * 9 + t, -1 after the last. A layer with more in
+// a channel, or an infinity or a NaN, needs w.
+// w: the weights as given, for the outputs that the split cannot give; null
+// in a network that parts and rests hold.
+struct WeightRest {
+    int index;
+    float value;
+};
+constexpr int kRests = 8;
+struct TowerWeights {
+    const float* parts;
+    const int* wexp;
+    const float* scale;   // folded BN
+    const float* shift;
+    const WeightRest* rest;
+    const float* w;
+};
+// Layers of such weights, one after the other `stride` words apart, each
+// array but w at its offset in the layer's.
+struct TowerLayers {
+    float* base;
+    const float* w;
+    size_t stride, wStride;
+    unsigned scale, shift, wexp, rest, parts;   // 32 bits: an address costs the kernels fewer scalar registers
+    __host__ __device__ TowerWeights at(int l) const {
+        const float* p = base + (size_t)l * stride;
+        return {p + parts,
+                reinterpret_cast<const int*>(p + wexp),
+                p + scale,
+                p + shift,
+                reinterpret_cast<const WeightRest*>(p + rest),
+                w ? w + (size_t)l * wStride : nullptr};
+    }
+};
 constexpr int kNoSplit = 1 << 20;
 __host__ __device__ constexpr bool hasSplit(int wexp) { return wexp < kNoSplit / 2; }
-size_t packedTowerFloats(int cin, int cout);
-hipError_t launchPackTower(const float* w, int cin, int cout, float* out, int* wexp, int layers, size_t stride,
+// The offsets and strides of a layer (base and w null): every array starts and
+// ends at a multiple of 64 words, the first three are zeros past cout.
+TowerLayers towerLayers(int cin, int cout);
+// Fills parts, wexp and rest of `layers` layers from layer `first` on, from
+// their weights w (one after the other) on the device. Sets *needsW where a
+// layer needs its weights as given.
+hipError_t launchPackTower(const TowerLayers& t, int first, int layers, const float* w, int cin, int cout, int* needsW,
                            hipStream_t stream);
 
 // How a convolution launch is cut: output channels per workgroup (a
@@ -151,9 +190,8 @@ template <int N, int COW, int WCO, int WPG, int PPW>
 hipError_t launchStemT(const float* x, const float* wp, const float* scale, const float* shift, const float* skip,
                        float* y, const BoardScales& s, int B, int cin, int cout, bool relu, hipStream_t stream);
 template <int N, int COW, int WCO, int WPG, int PPW>
-hipError_t launchTowerT(const float* x, const float* wp, const int* wexp, const float* scale, const float* shift,
-                        const float* skip, float* y, const BoardScales& s, int B, int cin, int cout, bool relu,
-                        hipStream_t stream);
+hipError_t launchTowerT(const float* x, const TowerWeights& w, const float* skip, float* y, const BoardScales& s, int B,
+                        int cin, int cout, bool relu, hipStream_t stream);
 
 // y[b][co][p] = relu?( (scale[co] * conv(x)[b][co][p] + shift[co]) (+ skip[b][co][p]) )
 // with each multiply and add rounded separately (BatchNorm2d::forwardInfer,
@@ -161,13 +199,12 @@ hipError_t launchTowerT(const float* x, const float* wp, const int* wexp, const 
 // src/network.cpp:264-271). skip may alias y (in-place residual).
 // y and skip in channel quads. The stem: x the network's input planes
 // [B][cin][n*n], weights as packConv3x3 packs them; the tower: x a trunk
-// activation in channel quads, weights as packTower packs them.
+// activation in channel quads.
 hipError_t launchStem(const float* x, const float* wPacked, const float* scale, const float* shift, const float* skip,
                       float* y, const BoardScales& s, int B, int n, int cin, int cout, bool relu, ConvTiling tiling,
                       hipStream_t stream);
-hipError_t launchTower(const float* x, const float* wPacked, const int* wexp, const float* scale, const float* shift,
-                       const float* skip, float* y, const BoardScales& s, int B, int n, int cin, int cout, bool relu,
-                       ConvTiling tiling, hipStream_t stream);
+hipError_t launchTower(const float* x, const TowerWeights& w, const float* skip, float* y, const BoardScales& s, int B,
+                       int n, int cin, int cout, bool relu, ConvTiling tiling, hipStream_t stream);
 bool conv3x3Supported(int boardSize);
 
 // The stem and the residual tower in one launch, each board resident in one
@@ -181,11 +218,7 @@ struct ResidentTower {
     int P;
     float* x;     // the trunk (channel quads), in place
     float* mid;   // the blocks' middle activations
-    // Tower layer l (conv1, conv2 of each block in turn): packed weights at
-    // w0 + l * stride, its BN scale and shift and its weights' powers of two
-    // scaleOff, shiftOff and wexpOff floats after them.
-    const float* w0;
-    size_t stride, scaleOff, shiftOff, wexpOff;
+    TowerLayers w;   // the tower's layers: conv1, conv2 of each block in turn
     int layers, B, F;
 };
 bool residentTowerSupported(int boardSize, int F, int P);

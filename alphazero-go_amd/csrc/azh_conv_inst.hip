@@ -20,8 +20,7 @@ template hipError_t launchStemT<AZH_CONV_N, kStem.coPerWave, kStem.wavesCo, kSte
     bool, hipStream_t);
 constexpr ConvTiling kTower = kTowerTilings[AZH_CONV_TILING];
 template hipError_t launchTowerT<AZH_CONV_N, kTower.coPerWave, kTower.wavesCo, kTower.wavesPg, kTower.pgPerWave>(
-    const float*, const float*, const int*, const float*, const float*, const float*, float*, const BoardScales&, int,
-    int, int, bool, hipStream_t);
+    const float*, const TowerWeights&, const float*, float*, const BoardScales&, int, int, int, bool, hipStream_t);
 #endif
 
 } // namespace azh

@@ -41,11 +41,9 @@ int deviceCUs();
 // The whole residual tower of a 5x5, 9x9 or 13x13 board of up to 64
 // channels (as LDS allows) in one launch, one workgroup per board with its
 // activations in LDS (azh_small_tower.hip): `layers` (even) convolutions on
-// trunk [B][ceil(F/4)][n*n] quads in place, layer l's packed weights at w0 +
-// l * layerStride floats and its BN scale and shift and its weights' powers
-// of two at scaleOff, shiftOff and wexpOff floats after them. The same bits
-// as the per-layer launches. smallTowerLdsBytes: the LDS a workgroup needs
-// (0 for other boards); launches need at most kSmallTowerMaxLds.
+// trunk [B][ceil(F/4)][n*n] quads in place, layer l's weights w.at(l). The
+// same bits as the per-layer launches. smallTowerLdsBytes: the LDS a workgroup
+// needs (0 for other boards); launches need at most kSmallTowerMaxLds.
 // With a stem, the launch first runs the stem convolution from the
 // network's input planes [B][planes][n*n] (its packed weights, BN scale and
 // shift) into the trunk, as conv3x3Stem does; without one (nullptr or in ==
@@ -70,9 +68,8 @@ struct SmallHeads {
     int V = 0;
 };
 size_t smallTowerLdsBytes(int n, int F, int planes, bool heads, int V);
-hipError_t launchSmallTower(float* trunk, const SmallStem* stem, const SmallHeads* heads, const float* w0,
-                            size_t layerStride, size_t scaleOff, size_t shiftOff, size_t wexpOff, int layers, int B, int n,
-                            int F, hipStream_t stream);
+hipError_t launchSmallTower(float* trunk, const SmallStem* stem, const SmallHeads* heads, const TowerLayers& w,
+                            int layers, int B, int n, int F, hipStream_t stream);
 // Workgroups of one convolution launch of shape t over B boards of
 // boardSize x boardSize with cout output channels (the launcher's grid).
 long convWorkgroups(ConvTiling t, int cout, int B, int boardSize);

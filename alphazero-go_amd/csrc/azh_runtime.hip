@@ -262,18 +262,37 @@ std::vector<TensorSpec> tensorSpec(const azh_netcfg& c) {
 
 // ---------------------------------------------------------------- weights
 
-struct ConvW {
+struct StemW {
     const float* w;   // packed MFMA fragments
     const float* scale;
     const float* shift;
-    const int* wexp;   // the tower's: packTower's powers of two (null for the stem)
+};
+
+// A device allocation released on scope exit.
+struct DeviceBuffer {
+    void* p = nullptr;
+    DeviceBuffer() = default;
+    explicit DeviceBuffer(size_t bytes) { allocate(bytes); }
+    ~DeviceBuffer() {
+        if (p) (void)hipFree(p);
+    }
+    DeviceBuffer(const DeviceBuffer&) = delete;
+    DeviceBuffer& operator=(const DeviceBuffer&) = delete;
+    void allocate(size_t bytes) {   // once
+        if (bytes) check(hipMalloc(&p, bytes), "hipMalloc");
+    }
+    template <class T>
+    T* as() const {
+        return static_cast<T*>(p);
+    }
 };
 
 struct DeviceWeights {
     float* arena = nullptr;
     size_t bytes = 0;
-    ConvW stem{};
-    std::vector<ConvW> conv1, conv2;
+    DeviceBuffer towerW;   // the tower's weights as given, where its parts do not hold them
+    StemW stem{};
+    azh::TowerLayers tower{};   // conv1, conv2 of each block in turn
     azh::HeadWeights heads{};
     ~DeviceWeights() {
         if (arena) (void)hipFree(arena);
@@ -286,8 +305,7 @@ size_t weightFloats(const azh_netcfg& c) {
     const Shape s(c);
     size_t f = 0;
     f += alignFloats(azh::packedConv3x3Floats(s.P, s.F)) + 2 * alignFloats(s.F);
-    f += (size_t)s.blocks * 2 *
-         (alignFloats(azh::packedTowerFloats(s.F, s.F)) + 2 * alignFloats(s.F) + alignFloats(s.F + 1));
+    f += (size_t)s.blocks * 2 * azh::towerLayers(s.F, s.F).stride;
     f += alignFloats(4 * s.F) + 2 * alignFloats(4);
     f += alignFloats(azh::headPolicyWTFloats(s.n)) + alignFloats(s.A1);
     f += alignFloats(azh::headFc1WTFloats(s.n, s.V)) + alignFloats(s.V) + alignFloats(s.V) + alignFloats(1);
@@ -455,67 +473,40 @@ private:
     std::ifstream in_;
 };
 
-// A device allocation released on scope exit (the synchronous kernel entry points).
-struct DeviceBuffer {
-    void* p = nullptr;
-    explicit DeviceBuffer(size_t bytes) {
-        if (bytes) check(hipMalloc(&p, bytes), "hipMalloc");
-    }
-    ~DeviceBuffer() {
-        if (p) (void)hipFree(p);
-    }
-    DeviceBuffer(const DeviceBuffer&) = delete;
-    DeviceBuffer& operator=(const DeviceBuffer&) = delete;
-    template <class T>
-    T* as() const {
-        return static_cast<T*>(p);
-    }
-};
-
-// Packs, folds and uploads checked tensors into one device arena.
+// Packs, folds and uploads checked tensors into one device arena: the tower's
+// layers first, then the stem and the heads (host).
 void uploadWeights(const azh_netcfg& c, const std::map<std::string, const float*>& given, DeviceWeights& dw) {
     const Shape s(c);
     auto T = [&](const std::string& name) { return given.at(name); };
 
-    std::vector<float> host(weightFloats(c), 0.0f);
+    azh::TowerLayers& tower = dw.tower = azh::towerLayers(s.F, s.F);
+    const size_t layers = (size_t)s.blocks * 2, towerFloats = layers * tower.stride;
+    std::vector<float> host(weightFloats(c) - towerFloats, 0.0f);
     size_t off = 0;
     auto take = [&](size_t floats) {
         const size_t o = off;
         off += alignFloats(floats);
         return o;
     };
-    struct ConvOff {
-        size_t w, scale, shift, wexp;
+    auto fold = [&](const std::string& bn, float* scale, float* shift) {
+        foldBn(T(bn + ".gamma"), T(bn + ".beta"), T(bn + ".runMean"), T(bn + ".runVar"), s.F, scale, shift);
     };
-    // The tower's weights, packed on the GPU once the rest is there.
-    std::vector<std::pair<const float*, ConvOff>> toPack;
-    auto fold = [&](ConvOff& o, const std::string& bn) {
-        o.scale = take(s.F);
-        o.shift = take(s.F);
-        foldBn(T(bn + ".gamma"), T(bn + ".beta"), T(bn + ".runMean"), T(bn + ".runVar"), s.F, &host[o.scale],
-               &host[o.shift]);
-    };
-    ConvOff stem{};
-    {
-        const std::vector<float> packed = azh::packConv3x3(T("stem.conv.w"), s.P, s.F);
-        stem.w = take(packed.size());
-        std::copy(packed.begin(), packed.end(), host.begin() + stem.w);
-        fold(stem, "stem.bn");
-    }
-    auto conv = [&](const std::string& wname, const std::string& bn) {
-        ConvOff o{};
-        o.w = take(azh::packedTowerFloats(s.F, s.F));
-        fold(o, bn);
-        o.wexp = take(s.F + 1);
-        toPack.push_back({T(wname), o});
-        return o;
-    };
-    std::vector<ConvOff> c1, c2;
-    for (int i = 0; i < s.blocks; ++i) {
-        const std::string p = "block" + std::to_string(i);
-        c1.push_back(conv(p + ".conv1.w", p + ".bn1"));
-        c2.push_back(conv(p + ".conv2.w", p + ".bn2"));
-    }
+    const std::vector<float> packed = azh::packConv3x3(T("stem.conv.w"), s.P, s.F);
+    const size_t stemW = take(packed.size()), stemScale = take(s.F), stemShift = take(s.F);
+    std::copy(packed.begin(), packed.end(), host.begin() + stemW);
+    fold("stem.bn", &host[stemScale], &host[stemShift]);
+    // The tower's layers: their weights, and their BN factors with the zeros
+    // up to the next array.
+    std::vector<const float*> towerW;
+    const size_t factors = tower.wexp - tower.scale;
+    std::vector<float> towerFactors(layers * factors, 0.0f);
+    for (int i = 0; i < s.blocks; ++i)
+        for (const char* h : {"1", "2"}) {
+            const std::string p = "block" + std::to_string(i);
+            float* f = &towerFactors[towerW.size() * factors];
+            fold(p + ".bn" + h, f, f + (tower.shift - tower.scale));
+            towerW.push_back(T(p + ".conv" + h + ".w"));
+        }
     // The heads' 1x1 rows: policy 0-1, value 2, ownership 3 (zero without the head).
     const size_t hConv = take(4 * s.F), hScale = take(4), hShift = take(4);
     std::copy(T("policy.conv.w"), T("policy.conv.w") + 2 * s.F, host.begin() + hConv);
@@ -546,54 +537,46 @@ void uploadWeights(const azh_netcfg& c, const std::map<std::string, const float*
     std::copy(T("value.fc2.w"), T("value.fc2.w") + s.V, host.begin() + f2W);
     host[f2B] = T("value.fc2.b")[0];
 
-    dw.bytes = host.size() * sizeof(float);
+    dw.bytes = (towerFloats + host.size()) * sizeof(float);
     check(hipMalloc(&dw.arena, dw.bytes), "hipMalloc(weights)");
-    // The arena but for the tower's packed weights: whole while it is small
-    // (its copies would cost more than their zeros), else a gap between them
-    // at a time.
-    constexpr size_t kSmall = size_t(4) << 20;
-    size_t from = 0;
-    auto upload = [&](size_t end) {
-        check(hipMemcpy(dw.arena + from, &host[from], (end - from) * sizeof(float), hipMemcpyHostToDevice),
+    auto upload = [&](float* dst, const float* src, size_t floats) {
+        check(hipMemcpy(dst, src, floats * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy(weights)");
+    };
+    // Rows of `row` floats, one per tower layer, `at` floats into it.
+    auto uploadRows = [&](size_t at, const float* src, size_t row) {
+        check(hipMemcpy2D(dw.arena + at, tower.stride * sizeof(float), src, row * sizeof(float), row * sizeof(float),
+                          layers, hipMemcpyHostToDevice),
               "hipMemcpy(weights)");
     };
-    if (dw.bytes > kSmall)
-        for (const auto& p : toPack) {
-            if (p.second.w > from) upload(p.second.w);
-            from = p.second.scale;
-        }
-    upload(host.size());
-    if (!toPack.empty()) {
+    upload(dw.arena + towerFloats, host.data(), host.size());
+    tower.base = dw.arena;
+    if (layers) {
+        uploadRows(tower.scale, towerFactors.data(), factors);
         // As many layers' weights at a time as kSmall holds, through one
         // device buffer (the null stream orders copies and kernels).
-        const size_t raw = (size_t)s.F * s.F * 9;
-        const size_t group = std::min(toPack.size(), std::max<size_t>(1, kSmall / (raw * sizeof(float))));
-        const size_t stride = toPack.size() > 1 ? toPack[1].second.w - toPack[0].second.w : 0;
+        constexpr size_t kSmall = size_t(4) << 20;
+        const size_t raw = tower.wStride;
+        const size_t group = std::min(layers, std::max<size_t>(1, kSmall / (raw * sizeof(float))));
         std::vector<float> staged(group > 1 ? group * raw : 0);
-        DeviceBuffer w(group * raw * sizeof(float));
-        for (size_t l = 0; l < toPack.size(); l += group) {
-            const size_t n = std::min(group, toPack.size() - l);
-            for (size_t i = 0; group > 1 && i < n; ++i)
-                std::copy(toPack[l + i].first, toPack[l + i].first + raw, staged.begin() + i * raw);
-            check(hipMemcpy(w.p, group > 1 ? staged.data() : toPack[l].first, n * raw * sizeof(float),
-                            hipMemcpyHostToDevice),
-                  "hipMemcpy(weights)");
-            check(azh::launchPackTower(w.as<float>(), s.F, s.F, dw.arena + toPack[l].second.w,
-                                       reinterpret_cast<int*>(dw.arena + toPack[l].second.wexp), (int)n, stride, nullptr),
+        DeviceBuffer w(group * raw * sizeof(float)), needsW(sizeof(int));
+        check(hipMemset(needsW.p, 0, sizeof(int)), "hipMemset(weights)");
+        for (size_t l = 0; l < layers; l += group) {
+            const size_t n = std::min(group, layers - l);
+            for (size_t i = 0; group > 1 && i < n; ++i) std::copy(towerW[l + i], towerW[l + i] + raw, &staged[i * raw]);
+            upload(w.as<float>(), group > 1 ? staged.data() : towerW[l], n * raw);
+            check(azh::launchPackTower(tower, (int)l, (int)n, w.as<float>(), s.F, s.F, needsW.as<int>(), nullptr),
                   "pack weights");
         }
-        check(hipStreamSynchronize(nullptr), "hipStreamSynchronize(weights)");
+        int needs = 0;
+        check(hipMemcpy(&needs, needsW.p, sizeof(int), hipMemcpyDeviceToHost), "hipMemcpy(weights)");
+        if (needs) {
+            dw.towerW.allocate(layers * raw * sizeof(float));
+            for (size_t l = 0; l < layers; ++l) upload(dw.towerW.as<float>() + l * raw, towerW[l], raw);
+            tower.w = dw.towerW.as<float>();
+        }
     }
-    const float* base = dw.arena;
-    auto mk = [&](const ConvOff& o) {
-        return ConvW{base + o.w, base + o.scale, base + o.shift,
-                     o.wexp ? reinterpret_cast<const int*>(base + o.wexp) : nullptr};
-    };
-    dw.stem = mk(stem);
-    for (int i = 0; i < s.blocks; ++i) {
-        dw.conv1.push_back(mk(c1[i]));
-        dw.conv2.push_back(mk(c2[i]));
-    }
+    const float* base = dw.arena + towerFloats;
+    dw.stem = StemW{base + stemW, base + stemScale, base + stemShift};
     dw.heads = azh::HeadWeights{base + hConv, base + hScale, base + hShift, base + pW, base + pB,
                                 base + f1W,   base + f1B,    base + f2W,    base + f2B};
 }
@@ -985,18 +968,12 @@ struct azh_runner {
     std::vector<std::unique_ptr<Slot>> slots;
     bool graphs = true;
     // The whole pass in one launch on small boards (azh::launchSmallTower):
-    // allowed (a test hook turns it off), and the tower convolutions' place
-    // in the weight arena (one fixed stride; `tower.ok` once checked).
+    // allowed (a test hook turns it off).
     bool smallTower = true;
     // The board-resident tower (azh::launchResidentTower): 0 never, 1 for a
     // pass alone on the device whose batch fills its rounds of CUs
     // (useResidentTower), 2 wherever the network allows it (a test hook).
     int residentTower = 1;
-    struct TowerLayout {
-        bool ok = false;
-        const float* w0 = nullptr;
-        size_t stride = 0, scaleOff = 0, shiftOff = 0, wexpOff = 0;
-    } tower;
 
     Reporter reporter;
     int device = 0;   // where the weights and slots live
@@ -1052,16 +1029,14 @@ struct azh_runner {
     int launchTowerOn(float* x, float* mid, Scales& sc, int Bp, azh::ConvTiling t, hipStream_t stream,
                       int blocksToRun) {
         const Shape& sh = shape;
-        auto layer = [&](const ConvW& c, const float* in, const float* skip, float* out, const char* what) {
+        auto layer = [&](int l, const float* in, const float* skip, float* out, const char* what) {
             const azh::BoardScales s{scaleBytes(sc, sc.now), outBytes(sc, t), sc.parts, scaleStride()};
-            check(azh::launchTower(in, c.w, c.wexp, c.scale, c.shift, skip, out, s, Bp, sh.n, sh.F, sh.F, true, t,
-                                   stream),
-                  what);
+            check(azh::launchTower(in, weights.tower.at(l), skip, out, s, Bp, sh.n, sh.F, sh.F, true, t, stream), what);
             advance(sc, t, out, Bp, stream);
         };
         for (int i = 0; i < blocksToRun; ++i) {
-            layer(weights.conv1[i], x, nullptr, mid, "conv3x3 (conv1)");
-            layer(weights.conv2[i], mid, x, x, "conv3x3 (conv2)");
+            layer(2 * i, x, nullptr, mid, "conv3x3 (conv1)");
+            layer(2 * i + 1, mid, x, x, "conv3x3 (conv2)");
         }
         return 2 * std::max(blocksToRun, 0);
     }
@@ -1127,8 +1102,8 @@ struct azh_runner {
                 hd.own = io.own;
                 hd.V = sh.V;
             }
-            check(azh::launchSmallTower(io.x, &stem, &hd, tower.w0, tower.stride, tower.scaleOff, tower.shiftOff,
-                                        tower.wexpOff, 2 * std::max(blocksToRun, 0), Bp, sh.n, sh.F, stream),
+            check(azh::launchSmallTower(io.x, &stem, &hd, weights.tower, 2 * std::max(blocksToRun, 0), Bp, sh.n, sh.F,
+                                        stream),
                   "small-board pass");
             return;
         }
@@ -1146,29 +1121,6 @@ struct azh_runner {
                   "heads");
     }
 
-    // Checks that the tower's convolutions sit in the weight arena at one
-    // fixed stride (conv1 and conv2 of each block in turn, each with its BN
-    // scale and shift at fixed offsets after its packed weights), as the
-    // small-board tower kernel reads them.
-    void initTowerLayout() {
-        const std::vector<ConvW>& c1 = weights.conv1;
-        const std::vector<ConvW>& c2 = weights.conv2;
-        tower = TowerLayout{};
-        if (c1.empty() || c2.size() != c1.size()) return;
-        const float* w0 = c1[0].w;
-        auto wexp = [](const ConvW& c) { return reinterpret_cast<const float*>(c.wexp); };
-        if (c2[0].w <= w0 || c1[0].scale < w0 || c1[0].shift < w0 || wexp(c1[0]) < w0) return;
-        const size_t stride = (size_t)(c2[0].w - w0), scaleOff = (size_t)(c1[0].scale - w0),
-                     shiftOff = (size_t)(c1[0].shift - w0), wexpOff = (size_t)(wexp(c1[0]) - w0);
-        for (size_t i = 0; i < c1.size(); ++i)
-            for (int h = 0; h < 2; ++h) {
-                const ConvW& c = h == 0 ? c1[i] : c2[i];
-                const float* w = w0 + (2 * i + h) * stride;
-                if (c.w != w || c.scale != w + scaleOff || c.shift != w + shiftOff || wexp(c) != w + wexpOff) return;
-            }
-        tower = TowerLayout{true, w0, stride, scaleOff, shiftOff, wexpOff};
-    }
-
     // Whether a pass of B runs as one small-board launch (stem, tower,
     // heads). A board's pass in one workgroup takes the same time up to a
     // board per CU, the per-layer launches a least time of 4-5 us a layer and
@@ -1180,7 +1132,7 @@ struct azh_runner {
     // channels at any batch (6x16: 53.3 / 74.3 at 8, 54.8 / 95.4 at 256) and
     // up to 32 past 16 boards (6x32: 69.2 / 77.1 at 17, 71.5 at 8 per layer).
     bool useSmallTower(int B) const {
-        if (!smallTower || !tower.ok) return false;
+        if (!smallTower || shape.blocks == 0) return false;
         const Shape& sh = shape;
         const size_t lds = azh::smallTowerLdsBytes(sh.n, sh.F, sh.P, true, sh.V);
         if (lds == 0 || lds > azh::kSmallTowerMaxLds) return false;
@@ -1205,8 +1157,7 @@ struct azh_runner {
     // pass's kernels (heads included) wait for them.
     bool useResidentTower(int B, bool alone) const {
         const Shape& sh = shape;
-        if (residentTower == 0 || (!tower.ok && sh.blocks > 0) || B < 1 ||
-            !azh::residentTowerSupported(sh.n, sh.F, sh.P))
+        if (residentTower == 0 || B < 1 || !azh::residentTowerSupported(sh.n, sh.F, sh.P))
             return false;
         if (residentTower == 2) return true;
         const long cus = azh::deviceCUs();
@@ -1229,11 +1180,7 @@ struct azh_runner {
         }
         t.x = io.x;
         t.mid = io.mid;
-        t.w0 = tower.w0;
-        t.stride = tower.stride;
-        t.scaleOff = tower.scaleOff;
-        t.shiftOff = tower.shiftOff;
-        t.wexpOff = tower.wexpOff;
+        t.w = weights.tower;
         t.layers = 2 * std::max(blocksToRun, 0);
         t.B = Bp;
         t.F = sh.F;
@@ -1322,9 +1269,8 @@ struct azh_runner {
             return;
         }
         if (useSmallTower(B)) {
-            check(azh::launchSmallTower(s.dX, nullptr, nullptr, tower.w0, tower.stride, tower.scaleOff,
-                                        tower.shiftOff, tower.wexpOff, 2 * std::max(blocksToRun, 0), B, shape.n,
-                                        shape.F, s.stream),
+            check(azh::launchSmallTower(s.dX, nullptr, nullptr, weights.tower, 2 * std::max(blocksToRun, 0), B,
+                                        shape.n, shape.F, s.stream),
                   "small-board tower");
             return;
         }
@@ -1508,7 +1454,6 @@ void createRunner(const azh_netcfg* cfg, const azh_tensor* tensors, int count, i
     scratchOnCurrentDevice();   // azh_infer_noalloc's scratch, resolved at set-up on the runner's device
     azh::deviceCUs();           // the launch rules' CU count, read once here, not during a caller's capture
     uploadWeights(*cfg, given, r->weights);
-    r->initTowerLayout();
     for (int i = 0; i < slots; ++i) r->slots.push_back(std::make_unique<Slot>(r->shape, max_batch));
     r->reporter.start();
     *out = r.release();
@@ -1637,33 +1582,56 @@ azh::ConvTiling probeTiling(bool planarIn, int tiling, int cout, int B, int n) {
     return planarIn ? azh::chooseStemTiling(cout, B, n, true) : azh::chooseTowerTiling(cout, B, n, true);
 }
 
-// The probes' weights on the device: the stem's packed ones, or the tower's,
-// packed there (with their powers of two, wexp).
-void probeWeights(bool planarIn, const std::vector<float>& packed, const float* w, int cin, int cout, float* dst,
-                  int* wexp) {
-    if (planarIn) {
-        check(hipMemcpy(dst, packed.data(), packed.size() * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
-        return;
-    }
-    const size_t raw = (size_t)cout * cin * 9 * sizeof(float);
-    DeviceBuffer d(raw);
-    check(hipMemcpy(d.p, w, raw, hipMemcpyHostToDevice), "hipMemcpy");
-    check(azh::launchPackTower(d.as<float>(), cin, cout, dst, wexp, 1, 0, nullptr), "pack weights");
-    check(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
-}
+// A probe's convolution on the device: the stem's from input planes, or the
+// tower's from channel quads.
+struct ProbeConv {
+    bool planar;
+    int n, cin, cout;
+    DeviceBuffer arena, given;
+    azh::TowerLayers tower;   // the stem's too: its packed weights, scale and shift
+    DeviceBuffer tops;        // a byte per board (BoardScales)
 
-// One convolution of the probes on the null stream: the stem's from input
-// planes, or the tower's from channel quads, whose scales it first scans
-// into dm (a byte per board).
-hipError_t probeConv(bool planarIn, const float* x, const float* w, const int* wexp, const float* scale,
-                     const float* shift, const float* skip, float* y, uint8_t* dm, int B, int n, int cin, int cout,
-                     bool relu, azh::ConvTiling t) {
-    const azh::BoardScales s{dm, nullptr, 1, 1};
-    if (planarIn) return azh::launchStem(x, w, scale, shift, skip, y, s, B, n, cin, cout, relu, t, nullptr);
-    const hipError_t e = azh::launchBoardScales(x, B, cin, n * n, dm, 1, nullptr);
-    if (e != hipSuccess) return e;
-    return azh::launchTower(x, w, wexp, scale, shift, skip, y, s, B, n, cin, cout, relu, t, nullptr);
-}
+    ProbeConv(bool planar, int B, int n, int cin, int cout, const float* w, const float* scale, const float* shift)
+        : planar(planar), n(n), cin(cin), cout(cout),
+          arena(planar ? (azh::packedConv3x3Floats(cin, cout) + 2 * alignFloats(cout)) * sizeof(float)
+                       : azh::towerLayers(cin, cout).stride * sizeof(float)),
+          tower(azh::towerLayers(cin, cout)), tops(B) {
+        tower.base = arena.as<float>();
+        auto upload = [&](size_t at, const float* src, size_t floats) {
+            check(hipMemcpy(tower.base + at, src, floats * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
+        };
+        if (planar) {
+            const std::vector<float> packed = azh::packConv3x3(w, cin, cout);
+            tower.scale = 0;
+            tower.shift = (unsigned)alignFloats(cout);
+            tower.parts = 2 * tower.shift;
+            upload(tower.parts, packed.data(), packed.size());
+        } else {
+            given.allocate(tower.wStride * sizeof(float));
+            DeviceBuffer needsW(sizeof(int));
+            check(hipMemset(needsW.p, 0, sizeof(int)), "hipMemset");
+            check(hipMemcpy(given.p, w, tower.wStride * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
+            check(azh::launchPackTower(tower, 0, 1, given.as<float>(), cin, cout, needsW.as<int>(), nullptr),
+                  "pack weights");
+            int needs = 0;
+            check(hipMemcpy(&needs, needsW.p, sizeof(int), hipMemcpyDeviceToHost), "hipMemcpy");
+            if (needs) tower.w = given.as<float>();
+        }
+        upload(tower.scale, scale, cout);
+        upload(tower.shift, shift, cout);
+    }
+    // Scans the input's magnitudes, for run().
+    void scan(const float* x, int B) {
+        if (!planar) check(azh::launchBoardScales(x, B, cin, n * n, tops.as<uint8_t>(), 1, nullptr), "board scales");
+    }
+    void run(const float* x, const float* skip, float* y, int B, bool relu, azh::ConvTiling t) {
+        const azh::TowerWeights w = tower.at(0);
+        const azh::BoardScales s{tops.as<uint8_t>(), nullptr, 1, 1};
+        check(planar ? azh::launchStem(x, w.parts, w.scale, w.shift, skip, y, s, B, n, cin, cout, relu, t, nullptr)
+                     : azh::launchTower(x, w, skip, y, s, B, n, cin, cout, relu, t, nullptr),
+              "conv3x3");
+    }
+};
 
 } // namespace
 
@@ -2175,7 +2143,7 @@ int azh_time_resident_tower(azh_runner* r, int slot, int B, int iters, int stem,
     return guarded([&] {
         if (!r || !ms || iters < 1) throw Error(AZH_ERR_ARGUMENT, "hip: bad timing arguments");
         const Shape& sh = r->shape;
-        if (!azh::residentTowerSupported(sh.n, sh.F, sh.P) || (!r->tower.ok && sh.blocks > 0))
+        if (!azh::residentTowerSupported(sh.n, sh.F, sh.P))
             throw Error(AZH_ERR_ARGUMENT, "hip: the board-resident tower does not take this network");
         r->checkBatch(B);
         const SlotClaim held = r->claimIdle(slot);
@@ -2247,39 +2215,17 @@ int azh_probe_conv3x3(const float* x, const float* w, const float* scale, const 
         // on the device gives that kernel.
         const bool planarIn = cin % azh::kChunk != 0;
         const azh::ConvTiling t = probeTiling(planarIn, tiling, cout, B, n);
-        const std::vector<float> packed = planarIn ? azh::packConv3x3(w, cin, cout) : std::vector<float>();
         const std::vector<float> xq = planarIn ? std::vector<float>() : azh::toChannelQuads(x, B, cin, (int)A);
         const std::vector<float> kq = skip ? azh::toChannelQuads(skip, B, cout, (int)A) : std::vector<float>();
         const size_t fx = planarIn ? B * cin * A : xq.size(), fy = azh::quadFloats(B, cout, (int)A);
-        std::vector<float*> bufs;
-        auto dev = [&](size_t floats) {
-            float* p = nullptr;
-            check(hipMalloc(&p, std::max<size_t>(floats, 1) * sizeof(float)), "hipMalloc");
-            bufs.push_back(p);
-            return p;
-        };
-        struct Free {
-            std::vector<float*>& b;
-            ~Free() {
-                for (float* p : b) (void)hipFree(p);
-            }
-        } guard{bufs};
-        float* dx = dev(fx);
-        float* dw = dev(planarIn ? packed.size() : azh::packedTowerFloats(cin, cout));
-        float* ds = dev(cout);
-        float* dh = dev(cout);
-        float* dy = dev(fy);
-        float* dk = skip ? dev(fy) : nullptr;
-        check(hipMemcpy(dx, planarIn ? x : xq.data(), fx * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
-        int* de = reinterpret_cast<int*>(dev(cout + 1));
-        uint8_t* dm = reinterpret_cast<uint8_t*>(dev(B));
-        probeWeights(planarIn, packed, w, cin, cout, dw, de);
-        check(hipMemcpy(ds, scale, cout * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
-        check(hipMemcpy(dh, shift, cout * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
-        if (dk) check(hipMemcpy(dk, kq.data(), fy * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
-        check(probeConv(planarIn, dx, dw, de, ds, dh, dk, dy, dm, B, n, cin, cout, relu != 0, t), "conv3x3");
+        ProbeConv conv(planarIn, B, n, cin, cout, w, scale, shift);
+        DeviceBuffer dx(fx * sizeof(float)), dy(fy * sizeof(float)), dk(kq.size() * sizeof(float));
+        check(hipMemcpy(dx.p, planarIn ? x : xq.data(), fx * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
+        if (skip) check(hipMemcpy(dk.p, kq.data(), fy * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
+        conv.scan(dx.as<float>(), B);
+        conv.run(dx.as<float>(), skip ? dk.as<float>() : nullptr, dy.as<float>(), B, relu != 0, t);
         std::vector<float> yq(fy);
-        check(hipMemcpy(yq.data(), dy, fy * sizeof(float), hipMemcpyDeviceToHost), "hipMemcpy");
+        check(hipMemcpy(yq.data(), dy.p, fy * sizeof(float), hipMemcpyDeviceToHost), "hipMemcpy");
         azh::fromChannelQuads(yq.data(), B, cout, (int)A, y);
     });
 }
@@ -2300,41 +2246,17 @@ int azh_time_conv3x3(int B, int n, int cin, int cout, int tiling, int iters, flo
             st = st * 1664525u + 1013904223u;
             v = ((st >> 8) * (1.0f / 16777216.0f) - 0.5f) * 0.05f;
         }
-        const std::vector<float> packed = planarIn ? azh::packConv3x3(w.data(), cin, cout) : std::vector<float>();
-        std::vector<float*> bufs;
-        struct Free {
-            std::vector<float*>& b;
-            ~Free() {
-                for (float* p : b) (void)hipFree(p);
-            }
-        } guard{bufs};
-        auto dev = [&](size_t floats) {
-            float* p = nullptr;
-            check(hipMalloc(&p, std::max<size_t>(floats, 1) * sizeof(float)), "hipMalloc");
-            bufs.push_back(p);
-            return p;
-        };
+        const std::vector<float> ones(cout, 1.0f), zeros(cout, 0.0f);
+        ProbeConv conv(planarIn, B, n, cin, cout, w.data(), ones.data(), zeros.data());
         const size_t fx = planarIn ? B * cin * A : azh::quadFloats(B, cin, (int)A);
-        float* dx = dev(fx);
-        float* dw = dev(planarIn ? packed.size() : azh::packedTowerFloats(cin, cout));
-        float* ds = dev(cout);
-        float* dh = dev(cout);
-        float* dy = dev(azh::quadFloats(B, cout, (int)A));
-        check(azh::launchFill(dx, fx, 0.5f, nullptr), "fill");
-        check(azh::launchFill(ds, cout, 1.0f, nullptr), "fill");
-        check(azh::launchFill(dh, cout, 0.0f, nullptr), "fill");
-        int* de = reinterpret_cast<int*>(dev(cout + 1));
-        uint8_t* dm = reinterpret_cast<uint8_t*>(dev(B));
-        probeWeights(planarIn, packed, w.data(), cin, cout, dw, de);
-        check(probeConv(planarIn, dx, dw, de, ds, dh, nullptr, dy, dm, B, n, cin, cout, true, t), "conv3x3");
+        DeviceBuffer dx(fx * sizeof(float)), dy(azh::quadFloats(B, cout, (int)A) * sizeof(float));
+        check(azh::launchFill(dx.as<float>(), fx, 0.5f, nullptr), "fill");
+        conv.scan(dx.as<float>(), B);
+        conv.run(dx.as<float>(), nullptr, dy.as<float>(), B, true, t);
         // A tower layer adds its input (here its own output); the stem adds
-        // nothing, as in the pass. dm holds the input's scales from the first
-        // launch.
+        // nothing, as in the pass.
         *ms = timeOnStream(nullptr, iters, [&] {
-            const azh::BoardScales s{dm, nullptr, 1, 1};
-            check(planarIn ? azh::launchStem(dx, dw, ds, dh, nullptr, dy, s, B, n, cin, cout, true, t, nullptr)
-                           : azh::launchTower(dx, dw, de, ds, dh, dy, dy, s, B, n, cin, cout, true, t, nullptr),
-                  "conv3x3");
+            conv.run(dx.as<float>(), planarIn ? nullptr : dy.as<float>(), dy.as<float>(), B, true, t);
         });
     });
 }

@@ -8,9 +8,9 @@ channel, three matrix products per pair, fp32 sums.
 - scaling a board or a channel's weights by a power of two scales the outputs
   by it, bit for bit, across the whole range of the scales: they only move
   exponents;
-- boards holding infinities or NaN, and layers with such weights, come out as
+- boards holding infinities or NaN, and channels with such weights, come out as
   the same products in fp32 give them, the same bits in every shape and in
-  every form of a pass, and other boards as without them.
+  every form of a pass, and other boards and channel blocks as without them.
 """
 import numpy as np
 import pytest
@@ -119,3 +119,71 @@ def test_infinite_inputs_same_bits_in_every_form(hip, cfg):
     for a, b, c in zip(one, per_layer, clean):
         assert bitwise_equal(a[rest], c[rest]) and bitwise_equal(b[rest], c[rest])
         assert np.array_equal(a[1], b[1], equal_nan=True)
+
+
+@pytest.mark.parametrize("n,F", [(5, 20), (9, 64), (13, 40), (19, 128)])
+def test_infinite_weight_stays_in_its_channel_block(hip, n, F):
+    """One infinite weight: the 16 channels of its block are summed from the
+    weights as given (channel 1's span 2^30, the large one on an input that is
+    zero, so that no rounding of it may show in the small ones' sums), the
+    others have the bits they have without it."""
+    F = -(-F // 16) * 16
+    x, w = _data(23 + n, n, F, F + 4, 2)
+    x[:, 0] = 0
+    w[1] *= np.float32(2.0 ** -30)
+    w[1, 4] = 1.0
+    clean = _raw(hip, x, w)
+    w[3, 5 * 9 + 4] = np.inf
+    with np.errstate(invalid="ignore"):
+        exact, mag = conv_exact_and_bound(x, w)
+    fin = np.isfinite(exact)
+    assert not fin[:, 3].any() and fin[:, :3].all()
+    outs = [_raw(hip, x, w, t) for t in TILINGS]
+    for o in outs:
+        assert np.array_equal(o, outs[0], equal_nan=True)
+        assert bitwise_equal(o[:, 16:], clean[:, 16:])
+        assert np.array_equal(np.isnan(o), np.isnan(exact)) and (o[np.isinf(exact)] == exact[np.isinf(exact)]).all()
+        assert (np.abs(o[fin] - exact[fin]) <= F * 9 * U * mag[fin]).all()
+
+
+@pytest.mark.parametrize("n,F", [(5, 16), (9, 64), (19, 144)])
+def test_few_weights_below_the_parts(hip, n, F):
+    """A channel whose sums are made by three weights 2^-30 of its largest, on
+    a board with an infinity in a corner: away from it the sums see every bit
+    of them, and the infinity meets them as it would the weights as given."""
+    x, w = _data(31 + n, n, F, F, 2)
+    x[:, 0] = 0
+    x[1, 2, 0] = np.inf
+    w[1] = 0
+    w[1, :9] = 1.0
+    for c, tap in ((1, 4), (5, 0), (F - 1, 8)):
+        w[1, c * 9 + tap] = np.float32(2.0 ** -30 * (1.1 + 0.3 * c))
+    w[2, 2 * 9 + 4] = np.float32(-2.0 ** -40)   # below both parts; meets the infinity
+    with np.errstate(invalid="ignore"):
+        exact, mag = conv_exact_and_bound(x, w)
+    fin = np.isfinite(exact)
+    assert exact[1, 2, 0] == -np.inf
+    outs = [_raw(hip, x, w, t) for t in TILINGS]
+    for o in outs:
+        assert np.array_equal(o, outs[0], equal_nan=True)
+        assert np.array_equal(np.isnan(o), np.isnan(exact)) and (o[np.isinf(exact)] == exact[np.isinf(exact)]).all()
+        assert (np.abs(o[1][fin[1]] - exact[1][fin[1]]) <= F * 9 * U * mag[1][fin[1]]).all()
+
+
+@pytest.mark.parametrize("cfg", [O.make_cfg(5, 2, 20), O.make_cfg(9, 2, 48), O.make_cfg(13, 2, 32),
+                                 O.make_cfg(19, 2, 128)])
+def test_infinite_weights_same_bits_in_every_form(hip, cfg):
+    net = O.random_network(cfg, 78)
+    t = net.tensors()
+    t["block0.conv2.w"][5 * 9 * cfg.filters + 4] = np.inf
+    t["block1.conv1.w"][2 * 9 * cfg.filters + 13] = -np.inf
+    B = 70 if cfg.board != 19 else 3
+    inp = np.random.default_rng(6).integers(0, 2, (B, cfg.planes, cfg.area)).astype(np.float32)
+    with hip.Runner(to_hip_cfg(hip, cfg), t, B, 1) as r:
+        r.set_resident_tower(2)
+        one = r.infer(inp)
+        r.set_resident_tower(0)
+        r.set_small_tower(False)
+        per_layer = r.infer(inp)
+    for a, b in zip(one, per_layer):
+        assert np.array_equal(a, b, equal_nan=True)
