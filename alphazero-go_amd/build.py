@@ -18,10 +18,11 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libazgo_hip.so")
 SOURCES = ["azh_kernels.hip", "azh_positions.hip", "azh_runtime.hip", "azh_small_tower.hip"]
 # The 3x3 convolution is one template instantiated per (board size,
-# workgroup shape): azh_conv_inst.hip is compiled once per pair, so the
-# fully unrolled kernels build in parallel.
+# workgroup shape, chunks of input channels): azh_conv_inst.hip is compiled
+# once for each, so the fully unrolled kernels build in parallel.
 CONV_INST = "azh_conv_inst.hip"
 CONV_HEADERS = ["azh_conv.hpp", "azh_conv_iface.hpp", "azh_resident.hpp", "azh_stem.hpp", "azh_tower.hpp", "azh_wave.hpp"]
+CONV_CHUNKS = (0, 1, 2)   # 0: three and more
 BOARD_SIZES = (5, 9, 13, 19)   # conv3x3Supported
 RESIDENT_BOARD_SIZES = (19,)   # residentTowerSupported
 HEADERS = CONV_HEADERS + ["azh_kernels.hpp", "azh_heads.hpp", os.path.join("..", "..", "include", "azgo_hip.h")]
@@ -78,7 +79,9 @@ def build(verbose=False, jobs=None, incremental=False):
     units = [(src, src.replace(".hip", ".o"), []) for src in SOURCES]
     for n in BOARD_SIZES:
         for t in range(conv_tiling_count()):
-            units.append((CONV_INST, f"azh_conv_{n}_{t}.o", [f"-DAZH_CONV_N={n}", f"-DAZH_CONV_TILING={t}"]))
+            for ch in CONV_CHUNKS:
+                units.append((CONV_INST, f"azh_conv_{n}_{t}_{ch}.o",
+                              [f"-DAZH_CONV_N={n}", f"-DAZH_CONV_TILING={t}", f"-DAZH_CONV_CH={ch}"]))
     for n in RESIDENT_BOARD_SIZES:
         units.append((CONV_INST, f"azh_resident_{n}.o", [f"-DAZH_CONV_N={n}", "-DAZH_RESIDENT_TOWER"]))
 

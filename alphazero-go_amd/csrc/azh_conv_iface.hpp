@@ -40,9 +40,13 @@ size_t packedConv3x3Floats(int cin, int cout);
 // fragments the kernel loads: [co block][chunk q][tap t][part h, l][lane
 // 0..63][j 0..7], value w[cb*16 + (lane & 15)][q*32 + 8*(lane >> 4) + j][t],
 // zero where the channel is padding (co blocks = packedCoBlocks(cout), chunks
-// = ceil(cin/32)) or the weight an infinity or a NaN.
-// wexp: cout powers of two, kNoSplit added for a channel with an infinity or
-// a NaN among its weights.
+// = ceil(cin/32); but the output channels that fill up the last quad repeat
+// its last one) or the weight an infinity or a NaN.
+// wexp: cout powers of two.
+// least: per channel, the magnitude a sum of the parts' products (that is,
+// 2^wexp and the activations' power of two in it) has to reach for what the
+// parts miss to be lost in its rounding (azh_tower.hpp); infinite for a
+// channel with an infinity or a NaN among its weights.
 // rest: of the weights that the parts miss by more than 2^-23 of them (2^-16
 // and less of the channel's largest), the difference: kRests a channel, in
 // the order of their index c * 9 + t, -1 after the last. A layer with more in
@@ -57,6 +61,7 @@ constexpr int kRests = 8;
 struct TowerWeights {
     const float* parts;
     const int* wexp;
+    const float* least;
     const float* scale;   // folded BN
     const float* shift;
     const WeightRest* rest;
@@ -68,23 +73,22 @@ struct TowerLayers {
     float* base;
     const float* w;
     size_t stride, wStride;
-    unsigned scale, shift, wexp, rest, parts;   // 32 bits: an address costs the kernels fewer scalar registers
+    unsigned scale, shift, wexp, least, rest, parts;   // 32 bits: an address costs the kernels fewer scalar registers
     __host__ __device__ TowerWeights at(int l) const {
         const float* p = base + (size_t)l * stride;
         return {p + parts,
                 reinterpret_cast<const int*>(p + wexp),
+                p + least,
                 p + scale,
                 p + shift,
                 reinterpret_cast<const WeightRest*>(p + rest),
                 w ? w + (size_t)l * wStride : nullptr};
     }
 };
-constexpr int kNoSplit = 1 << 20;
-__host__ __device__ constexpr bool hasSplit(int wexp) { return wexp < kNoSplit / 2; }
 // The offsets and strides of a layer (base and w null): every array starts and
-// ends at a multiple of 64 words, the first three are zeros past cout.
+// ends at a multiple of 64 words, the first four are zeros past cout.
 TowerLayers towerLayers(int cin, int cout);
-// Fills parts, wexp and rest of `layers` layers from layer `first` on, from
+// Fills parts, wexp, least and rest of `layers` layers from layer `first` on, from
 // their weights w (one after the other) on the device. Sets *needsW where a
 // layer needs its weights as given.
 hipError_t launchPackTower(const TowerLayers& t, int first, int layers, const float* w, int cin, int cout, int* needsW,
@@ -169,8 +173,8 @@ void fromChannelQuads(const float* quads, int B, int C, int A, float* planar);
 
 // A convolution hands the next one each board's largest magnitude, which
 // its operands' scale is made from (azh_tower.hpp): every wave writes the
-// biased exponent of its own outputs' largest (255: an infinity or a NaN) to
-// one byte, board b's wave i at bytes + b * stride + i.
+// biased exponent of its own outputs' largest (255: an infinity or a NaN; 0:
+// nothing but zeros) to one byte, board b's wave i at bytes + b * stride + i.
 struct BoardScales {
     const uint8_t* in;   // the input boards' (tower): inParts bytes each
     uint8_t* out;        // this layer's (null: not reported): convParts(shape) each
@@ -184,12 +188,13 @@ hipError_t launchBoardScales(const float* x, int B, int channels, int points, ui
                              hipStream_t stream);
 
 // One (board size, workgroup shape) instance of the stem's convolution
-// (azh_conv.hpp) and of the tower's (azh_tower.hpp), instantiated by
-// azh_conv_inst.hip, one object per shape.
+// (azh_conv.hpp) and of the tower's (azh_tower.hpp; CH: for one or two chunks
+// of input channels, 0: for more), instantiated by azh_conv_inst.hip, one
+// object per shape and CH.
 template <int N, int COW, int WCO, int WPG, int PPW>
 hipError_t launchStemT(const float* x, const float* wp, const float* scale, const float* shift, const float* skip,
                        float* y, const BoardScales& s, int B, int cin, int cout, bool relu, hipStream_t stream);
-template <int N, int COW, int WCO, int WPG, int PPW>
+template <int N, int COW, int WCO, int WPG, int PPW, int CH>
 hipError_t launchTowerT(const float* x, const TowerWeights& w, const float* skip, float* y, const BoardScales& s, int B,
                         int cin, int cout, bool relu, hipStream_t stream);
 

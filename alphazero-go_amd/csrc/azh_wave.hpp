@@ -23,11 +23,15 @@ __device__ __forceinline__ unsigned waveMax(unsigned v) {
     return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-// Writes the wave's byte for board b (BoardScales): the biased exponent of
-// its lanes' largest magnitude, top (bits).
+// The byte (BoardScales) of a largest magnitude (bits): its biased exponent,
+// at least 1 for anything but zero.
+__device__ __forceinline__ unsigned scaleByte(unsigned top) { return top ? max(top >> 23, 1u) : 0u; }
+
+// Writes the wave's byte for board b (BoardScales) of its lanes' largest
+// magnitude, top (bits).
 __device__ __forceinline__ void reportScale(const BoardScales& s, unsigned top, int b, int part) {
     top = waveMax(top);
-    if (s.out && (threadIdx.x & 63) == 0) s.out[(size_t)b * s.stride + part] = (uint8_t)(top >> 23);
+    if (s.out && (threadIdx.x & 63) == 0) s.out[(size_t)b * s.stride + part] = (uint8_t)scaleByte(top);
 }
 
 } // namespace

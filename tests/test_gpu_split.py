@@ -8,6 +8,8 @@ channel, three matrix products per pair, fp32 sums.
 - scaling a board or a channel's weights by a power of two scales the outputs
   by it, bit for bit, across the whole range of the scales: they only move
   exponents;
+- a value far above the rest of its board, or a weight far above the rest of
+  its channel's, costs the sums that do not see it no precision;
 - boards holding infinities or NaN, and channels with such weights, come out as
   the same products in fp32 give them, the same bits in every shape and in
   every form of a pass, and other boards and channel blocks as without them.
@@ -75,6 +77,68 @@ def test_powers_of_two_only_move_exponents(hip, kx, kw):
     assert np.isfinite(want).all() and bitwise_equal(got, want)
 
 
+def _fp32_grade(got, exact, mag, K):
+    """Within the bound of any fp32 order, and as close as the fp32 matrix
+    units' sums of random terms: K / 4 additions that each round a partial sum,
+    the partial sums no larger than the whole, in quadrature."""
+    err = np.abs(got.astype(np.float64) - exact)
+    assert (err <= K * U * mag).all()
+    rms = np.sqrt((err ** 2).mean() / (exact ** 2).mean())
+    assert rms <= U * np.sqrt(K / 4), f"{rms:.2e} of the sums"
+
+
+@pytest.mark.parametrize("spread", [8, 14, 17, 20, 24, 30, 40, 90])
+@pytest.mark.parametrize("n,F", [(5, 16), (9, 64), (13, 32), (19, 144)])
+def test_a_value_far_above_its_board(hip, n, F, spread):
+    """One activation 2^spread times the others' scale: the sums whose window
+    does not hold it, and the other boards', are as good as without it."""
+    x, w = _data(41 + n, n, F, F, 2)
+    clean = _raw(hip, x, w)
+    at = (n // 2) * n + n // 2
+    x[1, F // 2, at] = np.float32(2.0 ** spread)
+    exact, mag = conv_exact_and_bound(x, w)
+    rows, cols = np.divmod(np.arange(n * n), n)
+    away = (np.abs(rows - n // 2) > 1) | (np.abs(cols - n // 2) > 1)
+    outs = [_raw(hip, x, w, t) for t in TILINGS]
+    for o in outs[1:]:
+        assert bitwise_equal(o, outs[0])
+    assert bitwise_equal(outs[0][0], clean[0])
+    _fp32_grade(outs[0][1][:, away], exact[1][:, away], mag[1][:, away], F * 9)
+    assert (np.abs(outs[0][1] - exact[1]) <= F * 9 * U * mag[1]).all()
+
+
+@pytest.mark.parametrize("spread", [8, 14, 17, 20, 24, 30, 40, 90])
+@pytest.mark.parametrize("n,F", [(9, 64), (19, 128)])
+@pytest.mark.parametrize("few", [False, True])
+def test_a_weight_far_above_its_channel(hip, n, F, spread, few):
+    """One weight 2^spread times the others of its channel, on an input that is
+    zero; few: all but five of the others are zero."""
+    x, w = _data(43 + n, n, F, F, 2)
+    x[:, 5] = 0
+    if few:
+        w[3] = 0
+        w[3, 11::2 * F] = 0.01 + np.arange(5, dtype=np.float32) / 97
+    w[3, 5 * 9 + 4] = np.float32(2.0 ** spread)
+    exact, mag = conv_exact_and_bound(x, w)
+    outs = [_raw(hip, x, w, t) for t in TILINGS]
+    for o in outs[1:]:
+        assert bitwise_equal(o, outs[0])
+    _fp32_grade(outs[0][:, 3], exact[:, 3], mag[:, 3], F * 9)
+    rest = np.delete(np.arange(F), 3)
+    _fp32_grade(outs[0][:, rest], exact[:, rest], mag[:, rest], F * 9)
+
+
+def test_boards_of_zeros_and_of_denormals(hip):
+    x, w = _data(47, 9, 32, 32, 3)
+    x[0] = 0
+    x[1] *= np.float32(2.0 ** -122)
+    outs = [_raw(hip, x, w, t) for t in TILINGS]
+    exact, mag = conv_exact_and_bound(x, w)
+    for o in outs:
+        assert bitwise_equal(o, outs[0]) and not o[0].any()
+        assert (np.abs(o - exact) <= 32 * 9 * (U * mag + 2.0 ** -149)).all()
+
+
 @pytest.mark.parametrize("n,F", [(5, 16), (9, 64), (19, 128)])
 def test_infinities_and_nan(hip, n, F):
     B = 3
@@ -100,15 +164,16 @@ def test_infinities_and_nan(hip, n, F):
 
 @pytest.mark.parametrize("cfg", [O.make_cfg(5, 2, 20), O.make_cfg(9, 2, 48), O.make_cfg(13, 1, 32),
                                  O.make_cfg(19, 2, 128)])
-def test_infinite_inputs_same_bits_in_every_form(hip, cfg):
-    """Positions of which one holds an infinity: the one-launch forms (a board
+@pytest.mark.parametrize("value", [np.inf, 2.0 ** 22, 2.0 ** 60])
+def test_infinite_inputs_same_bits_in_every_form(hip, cfg, value):
+    """Positions of which one holds an infinity, or a value far above the rest: the one-launch forms (a board
     in LDS, a board resident) and the per-layer launches agree bit for bit,
     and the other positions are untouched."""
     net = O.random_network(cfg, 77)
     B = 70 if cfg.board != 19 else 3
     inp = np.random.default_rng(5).integers(0, 2, (B, cfg.planes, cfg.area)).astype(np.float32)
     bad = inp.copy()
-    bad[1, 0, 3] = np.inf
+    bad[1, 0, 3] = value
     with hip.Runner(to_hip_cfg(hip, cfg), net.tensors(), B, 1) as r:
         r.set_resident_tower(2)
         clean, one = r.infer(inp), r.infer(bad)
