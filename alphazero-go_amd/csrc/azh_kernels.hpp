@@ -48,7 +48,7 @@ int deviceCUs();
 // network's input planes [B][planes][n*n] (its packed weights, BN scale and
 // shift) into the trunk, as conv3x3Stem does; without one (nullptr or in ==
 // nullptr) it reads the trunk.
-constexpr size_t kSmallTowerMaxLds = 80 * 1024;   // two workgroups per CU
+constexpr size_t kSmallTowerMaxLds = 80 * 1024;   // two workgroups of a CU's 160 KB, all they declare counted
 constexpr int kSmallTowerMaxBlocks = 4;   // up to 64 channels: a block of 16 per wave
 struct SmallStem {
     const float* in = nullptr;

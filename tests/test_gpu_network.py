@@ -254,6 +254,8 @@ def test_small_board_split_boundaries(hip, tag, B):
     (O.make_cfg(5, 2, 32, history=1), 5),     # 4 input planes: one short chunk
     (O.make_cfg(9, 2, 32, history=7), 8),     # 16: one whole chunk, no short one
     (O.make_cfg(9, 2, 32, history=16), 9),    # 34: two whole chunks and 2 planes
+    (O.make_cfg(13, 2, 16, history=16), 7),   # over 64 KB of LDS
+    (O.make_cfg(9, 1, 64, history=47), 65),   # 96 planes: almost the 80 KB that are allowed
 ])
 def test_small_tower_equals_per_layer_launches(hip, cfg, B):
     """A small board's tower in one launch (one workgroup per board, the
