@@ -145,20 +145,21 @@ def test_headline_batch_independent(hip):
             assert bitwise_equal(part[0], whole[0][picks]) and bitwise_equal(part[1], whole[1][picks])
 
 
-@pytest.mark.parametrize("B", [257, 75, 21, 17])
+@pytest.mark.parametrize("B", [257, 113, 128, 75, 21, 17])
 def test_split_pass_equals_whole(hip, B):
-    """A batch with more than a round of workgroups, or a small one in the
-    four-wave shape of 6 column groups, runs as two half-batch chains on two
-    streams (forked and joined inside the captured graph), each half in its
-    own batch's shape: an odd batch (257: whole-board workgroups; 75: the
-    four-wave shape; 21: halves of 11 and 10 in a 2-group shape; 17: halves
-    of 9 and 8 in two different shapes), captured and eager, gives every row
-    the bits of the position alone, on both sides of the split."""
+    """A batch whose whole-board workgroups come to 7/8 of a round and more
+    runs as two half-batch chains on two streams (forked and joined inside the
+    captured graph), both halves in the batch's shape (on the MI355X 257, 113
+    and 128 boards; the smaller batches run as one chain): captured and eager,
+    it gives every row the bits of the position alone, on both sides of the
+    split."""
     w = O.WORKLOADS[3]
     net = O.random_network(w.cfg, 605)
     inp, _ = O.workload_inputs(w, B)
     half = (B + 1) // 2
     with _runner(hip, net, B) as r:
+        if hip.device_cus() == 256:
+            assert r.pass_form(B) == (r.FORM_SPLIT if B > 112 else 0)
         graph = r.infer(inp)
         again = r.infer(inp)
         assert bitwise_equal(again[0], graph[0]) and bitwise_equal(again[1], graph[1])
@@ -205,13 +206,18 @@ def test_graph_cache_eviction_keeps_the_bits(hip):
             assert bitwise_equal(again[0], want[0]) and bitwise_equal(again[1], want[1]), B
 
 
+def _form_changes(r, most, alone=True):
+    """The batches at which a pass's form changes, and the ones before them."""
+    forms = [r.pass_form(b, alone) for b in range(1, most + 1)]
+    return sorted({b for i in range(1, most) if forms[i] != forms[i - 1] for b in (i, i + 1)})
+
+
 @pytest.mark.parametrize("B", [5, 6, 8, 9, 16, 17, 18, 28, 29, 32, 33, 34, 115, 116, 128, 129, 217, 218])
 def test_shape_and_split_boundaries(hip, B):
-    """19x19 10x128 on both sides of each change of workgroup shape, of the
-    two-chain split and of the halves' own shapes (17: halves of 9 and 8
-    boards in two different shapes; 17-28 and 33: halves in a finer shape
-    than the batch's): rows at the start, the middle and the end are the
-    bits of their positions alone."""
+    """19x19 10x128 over the batches in which the workgroup shapes change,
+    the split (112 and 193 boards on the MI355X) and the board-resident launch
+    (129) begin: rows at the start, the middle and the end are the bits of
+    their positions alone."""
     w = O.WORKLOADS[3]
     net = O.random_network(w.cfg, 607)
     inp, _ = O.workload_inputs(w, B)
@@ -222,21 +228,73 @@ def test_shape_and_split_boundaries(hip, B):
             assert bitwise_equal(alone[0][0], whole[0][s]) and bitwise_equal(alone[1][0], whole[1][s]), s
 
 
-@pytest.mark.parametrize("tag,B", [(2, 128), (2, 129), (2, 191), (2, 192), (1, 1085), (1, 1086)])
+@pytest.mark.parametrize("cfg,most,changes", [
+    (O.make_cfg(19, 2, 128), 260, [111, 112, 128, 129, 192, 193]),
+    (O.make_cfg(9, 2, 64), 256, [223, 224]),
+    (O.make_cfg(13, 2, 90), 130, [37, 38, 42, 43, 111, 112, 128, 129]),
+    (O.make_cfg(5, 2, 32), 1100, [1085, 1086]),
+])
+def test_per_layer_split_boundaries(hip, cfg, most, changes):
+    """The per-layer launches on both sides of every batch at which they begin
+    or end to run as two half-batch chains (5x5 4x32: at the least layer work
+    that splits, 0.5 GFLOP): rows on both sides of the halves are the bits of
+    their positions alone."""
+    net = O.random_network(cfg, 608)
+    inp, _ = O.workload_inputs(O.Workload(0, "split", cfg, most, 0.3, 0.3), most)
+    with _runner(hip, net, most) as r:
+        r.set_small_tower(False)
+        r.set_resident_tower(0)
+        at = _form_changes(r, most)
+        if hip.device_cus() == 256:
+            assert at == changes
+        alone = {}
+        for B in at:
+            assert r.pass_form(B) in (0, r.FORM_SPLIT)
+            whole = r.infer(inp[:B])
+            for s in (0, (B - 1) // 2, (B + 1) // 2, B - 1):
+                if s not in alone:
+                    alone[s] = r.infer(inp[s:s + 1])
+                assert bitwise_equal(alone[s][0][0], whole[0][s]) and bitwise_equal(alone[s][1][0], whole[1][s]), (B, s)
+
+
+@pytest.mark.parametrize("tag,B", [(2, 128), (2, 129), (2, 191), (2, 192), (1, 1085), (1, 1086), (2, 64), (2, 65),
+                                   (2, 257), (1, 257)])
 def test_small_board_split_boundaries(hip, tag, B):
-    """9x9 6x64 around the smaller shapes' split (two chains past two rounds
-    of workgroups, from 129 boards) and the change to whole-board
-    workgroups at 192 boards (one chain again); 5x5 4x32 around the least
-    layer work that splits (0.5 GFLOP, from 1086 boards): rows on both
-    sides of the halves are the bits of their positions alone."""
+    """9x9 6x64 per layer up to 64 boards and in one launch past them, and 5x5
+    4x32, up to a board per CU and past it: rows at the start, the middle and
+    the end are the bits of their positions alone."""
     w = O.WORKLOADS[tag]
     net = O.random_network(w.cfg, 608)
     inp, _ = O.workload_inputs(w, B)
     with _runner(hip, net, B) as r:
+        assert r.pass_form(B) == (r.FORM_SMALL if tag == 1 or B > 64 else 0)
         whole = r.infer(inp)
         for s in (0, (B - 1) // 2, (B + 1) // 2, B - 1):
             alone = r.infer(inp[s:s + 1])
             assert bitwise_equal(alone[0][0], whole[0][s]) and bitwise_equal(alone[1][0], whole[1][s]), s
+
+
+# Past a board per CU the launch runs four waves a board where they cover its
+# column groups: their own split of the groups, idle waves (three channel
+# blocks) and sharing of the scale. One board with a value far above the
+# rest, one with an infinity: fragments summed again, and whole boards.
+@pytest.mark.parametrize("n,F", [(5, 48), (5, 64), (9, 16), (9, 20), (9, 32), (13, 12), (13, 16), (9, 64)])
+def test_small_tower_past_a_board_per_cu(hip, n, F):
+    cfg = O.make_cfg(n, 2, F)
+    B = hip.device_cus() + 5
+    net = O.random_network(cfg, 615)
+    inp, _ = O.workload_inputs(O.Workload(0, "four", cfg, B, 0.3, 0.3), B)
+    inp = inp.copy()
+    inp[2, 0, n + 1] = np.float32(2.0 ** 22)
+    inp[B - 1, 1, 3] = np.inf
+    with _runner(hip, net, B) as r:
+        assert r.pass_form(B) == r.FORM_SMALL
+        one = r.infer(inp)
+        few = r.infer(inp[:6])   # eight waves a board
+        r.set_small_tower(False)
+        per_layer = r.infer(inp)
+    for a, b, c in zip(one, per_layer, few):
+        assert np.array_equal(a, b, equal_nan=True) and np.array_equal(a[:6], c, equal_nan=True)
 
 
 @pytest.mark.parametrize("cfg,B", [
@@ -324,10 +382,11 @@ def test_resident_tower_mode_refused(hip):
 def test_pass_forms(hip):
     """How a pass runs, from the device's compute units (C): the
     board-resident tower for a pass alone whose batch gives one workgroup to
-    95% of the CUs (one round) or to every CU in each of several rounds;
-    otherwise, and beside another pass, the per-layer launches (on the
-    MI355X's 256 CUs in half-batch chains there); the small-board pass in one
-    launch on 9x9 at 64 channels past 128 boards."""
+    more than half of the CUs (towers of up to three blocks: to 95%) or to
+    every CU in each of several rounds; otherwise, and beside another pass, the
+    per-layer launches (on the MI355X's 256 CUs in half-batch chains there);
+    the small-board pass in one launch on 9x9 at 64 channels past 64 boards, on
+    13x13 at 32 channels past 16."""
     cus = hip.device_cus()
     one_round = -(-19 * cus // 20)   # the fewest boards that give one workgroup to 95% of the CUs
     net = O.random_network(O.make_cfg(19, 2, 128), 613)
@@ -352,9 +411,24 @@ def test_pass_forms(hip):
         r.input(0)[:cus] = O.workload_inputs(O.Workload(0, "forms", net.cfg, cus, 0.3, 0.3), cus)[0]
         r.stage(0, cus)
         assert r.time_resident_tower(0, cus, 2) > 0 and r.time_resident_tower(0, cus, 2, stem=False) > 0
+    net4 = O.random_network(O.make_cfg(19, 4, 128), 613)
+    with _runner(hip, net4, cus + 1) as r:
+        assert not r.pass_form(cus // 2) & r.FORM_RESIDENT
+        assert r.pass_form(cus // 2 + 1) == r.FORM_RESIDENT and r.pass_form(cus) == r.FORM_RESIDENT
+        assert not r.pass_form(cus + 1) & r.FORM_RESIDENT
+        assert not r.pass_form(cus // 2 + 1, alone=False) & r.FORM_RESIDENT
+        # The bits on both sides of the line.
+        inp = O.workload_inputs(O.Workload(0, "forms", net4.cfg, cus // 2 + 1, 0.3, 0.3), cus // 2 + 1)[0]
+        below, above = r.infer(inp[:-1]), r.infer(inp)
+        for a, b in zip(below, above):
+            assert bitwise_equal(a, b[:-1])
     net9 = O.random_network(O.make_cfg(9, 1, 64), 614)
     with _runner(hip, net9, 256) as r:
         assert r.pass_form(256) == r.FORM_SMALL
+        assert r.pass_form(64) == 0 and r.pass_form(65) == r.FORM_SMALL
+    net13 = O.random_network(O.make_cfg(13, 1, 32), 614)
+    with _runner(hip, net13, 17) as r:
+        assert r.pass_form(16) == 0 and r.pass_form(17) == r.FORM_SMALL
 
 
 @pytest.mark.parametrize("history,B", [(8, 256), (7, 256), (9, 256), (16, 256), (8, 40), (3, 5)])
