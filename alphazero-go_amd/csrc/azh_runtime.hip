@@ -1124,13 +1124,14 @@ struct azh_runner {
     // Whether a pass of B runs as one small-board launch (stem, tower,
     // heads). A board's pass in one workgroup takes the same time up to a
     // board per CU, the per-layer launches a least time of 4-5 us a layer and
-    // more with the batch. Per pass, one launch against per layer: 5x5 up to
-    // 64 channels at any batch (4x32: 23.9 against 45.7 us at 8 boards, 24.5
-    // against 58.3 at 256); 9x9 up to 32 channels at any batch (6x32: 49.7 /
-    // 68.9 at 8, 51.1 / 91.8 at 256) and up to 64 past 64 boards (6x64: 92.0
-    // / 114 at 65, 92.3 / 110 at 128; about 91 / 80 at 32); 13x13 up to 16
-    // channels at any batch (6x16: 53.3 / 74.3 at 8, 54.8 / 95.4 at 256) and
-    // up to 32 past 16 boards (6x32: 69.2 / 77.1 at 17, 71.5 at 8 per layer).
+    // more with the batch. us per pass of six blocks, per layer / one launch:
+    // 5x5 up to 64 channels at any batch; 9x9 up to 32 channels at any batch
+    // and up to 64 past 64 boards (36 channels, 65 boards 94.9 / 79.0; 48
+    // channels, 65 boards 93.4 / 79.4, 85 96.0 / 79.1; 64 channels, 65 boards
+    // 107.7 / 89.1; at 33 to 49 boards the one launch, forced, gains nothing);
+    // 13x13 up to 16 channels at any batch and up to 32 past 16 boards (20
+    // channels, 17 boards 69.3 / 66.0, 33 75.6 / 66.2; 32 channels, 17 boards
+    // 69.7 / 66.3, 33 76.5 / 66.5). The two lines are those of 256 CUs.
     bool useSmallTower(int B) const {
         if (!smallTower || shape.blocks == 0) return false;
         const Shape& sh = shape;
@@ -1148,13 +1149,15 @@ struct azh_runner {
     // round of workgroups idles CUs for all of it, while the per-layer
     // launches shrink with the batch, down to a round of half-board tiles at
     // half as many boards as CUs. So taken past those for one round, and for
-    // more rounds only when they are full. 19x19 10x128, us per pass,
-    // board-resident against per layer: 112 boards 1095 / 759, 129 1149 /
-    // 1285, 181 1206 / 1377, 242 1291 / 1565. Short towers gain less (one
-    // block: 129 boards 178 / 179, 160 184 / 182, 200 186 / 203): up to three
-    // blocks from 95% of the CUs. Not with another pass in flight: its
-    // workgroups hold every CU's registers for a whole tower, so the other
-    // pass's kernels (heads included) wait for them.
+    // more rounds only when they are full. 19x19, 128 channels, us per pass,
+    // per layer / board-resident: ten blocks 112 boards 759 / 1095, 129 1285 /
+    // 1149, 242 1565 / 1291; six 129 820 / 665, 242 971 / 756; four 129 566 /
+    // 470. Up to three blocks the line is still the fp32 tower's, 95% of the
+    // CUs, though this launch is the faster one from 129 boards on there too
+    // (three blocks 129 boards 439 / 376, 242 518 / 417; two 312 / 278, 373 /
+    // 308; one 184 / 173, 225 / 195); so it is with another pass in flight,
+    // where it is not taken (two slots kept full, 256 boards a pass: 175 k
+    // positions/s per layer, 190 k with it forced).
     bool useResidentTower(int B, bool alone) const {
         const Shape& sh = shape;
         if (residentTower == 0 || B < 1 || !azh::residentTowerSupported(sh.n, sh.F, sh.P))

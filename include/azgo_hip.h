@@ -18,6 +18,14 @@
  * inference_batch"). Arrays are fp32, row-major, the reference's layouts:
  * input [B][2H+2][n*n] (Evaluator::evaluate, include/azgo/evaluator.hpp:24),
  * logits [B][n*n+1], values [B] (tanh).
+ *
+ * Arithmetic: fp32 throughout but for the residual tower's convolutions, which
+ * multiply each fp32 operand as two f16 parts (three products a pair, fp32
+ * sums) under a power of two per board and layer and per output channel. Sums
+ * too small for what such parts hold, and those of boards or channels with an
+ * infinity or a NaN, are made again from the fp32 operands, so that the error
+ * stays an fp32 sum's whatever the range of the values. A position's bits
+ * depend neither on its batch nor on how the pass runs.
  */
 #ifndef AZGO_HIP_H
 #define AZGO_HIP_H
@@ -393,7 +401,7 @@ int azh_time_pipelined_positions(azh_runner* r, const azh_positions* pos, int B,
  * groups per wave; 0 = the board's, shared by the waves): the tower's
  * 0 (2,4,2,0), 1 (2,2,4,0), 2 (2,1,4,0), 3 (1,1,4,0), 4 (2,2,2,0),
  * 5 (2,2,4,3), 6 (2,1,4,3), 7 (1,2,4,3), 8 (1,2,3,2), 9 (1,1,3,2),
- * 10 (1,1,6,1), 11 (1,1,3,1), 12 (1,2,3,1); the stem's 0 (2,2,2,12),
+ * 10 (1,1,1,1), 11 (1,1,3,1), 12 (1,2,3,1); the stem's 0 (2,2,2,12),
  * 1 (1,4,1,0), 2 (1,2,1,0), 3 (1,1,1,0), 4 (1,8,1,0), 5 (1,2,2,12),
  * 6 (1,1,4,6), 7 (1,1,4,2), 8 (1,1,4,1), 9 (1,1,8,1), 10 (1,1,3,1),
  * 11 (1,1,6,1), 12 (1,1,6,2). */
