@@ -575,6 +575,8 @@ void uploadWeights(const azh_netcfg& c, const std::map<std::string, const float*
             tower.w = dw.towerW.as<float>();
         }
     }
+    // The runner's streams do not wait for the null stream's copies.
+    check(hipStreamSynchronize(nullptr), "hipStreamSynchronize(weights)");
     const float* base = dw.arena + towerFloats;
     dw.stem = StemW{base + stemW, base + stemScale, base + stemShift};
     dw.heads = azh::HeadWeights{base + hConv, base + hScale, base + hShift, base + pW, base + pB,

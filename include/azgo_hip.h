@@ -106,7 +106,10 @@ const char* azh_last_error(void);
 
 /* checkCudaInferenceMemory / hubBytes (include/azgo/cuda.hpp:60-66;
  * src/cuda/cuda_runner.cu:186-223): device bytes one runner of `slots` slots
- * of max_batch positions needs (weights included). */
+ * of max_batch positions needs (weights included; not the copy of its tower's
+ * fp32 weights that a network keeps when one of them is not finite, or more
+ * than eight of an output channel are under 2^-16 of its largest and not held
+ * by two f16 parts). */
 int azh_memory_need(const azh_netcfg* cfg, int max_batch, int slots, size_t* bytes);
 
 /* The same check the constructor makes: AZH_ERR_MEMORY with the reference's
